@@ -156,6 +156,7 @@ __global__ __launch_bounds__(kThreads, MINW) void fwd_uniform_kernel(const float
     Hit h;
     wh.load(l, h);
     Trk prop;
+    float r;
     if (SEM == P2R_REFERENCE) {
       // tbb.cpp:894: every layer starts from the input track.  The barriers, on the input parameters in
       // place and on the covariance column's offset, make every layer recompute and reread it; nothing is
@@ -166,11 +167,11 @@ __global__ __launch_bounds__(kThreads, MINW) void fwd_uniform_kernel(const float
       asm volatile("" : "+v"(col));
       q = q_in;
       k = (float)q * kfact;
-      Lane<EXACT>::propagate(in_par, LdsCov{cov_lds + col * 21u}, k, h.pos[0], h.pos[1], prop);
+      r = Lane<EXACT>::propagate(in_par, LdsCov{cov_lds + col * 21u}, k, h.pos[0], h.pos[1], prop);
     } else {
-      Lane<EXACT>::propagate(cur, k, h.pos[0], h.pos[1], prop);  // propagate-tor-test_hip.cu:842-845
+      r = Lane<EXACT>::propagate(cur.par, cur.cov, k, h.pos[0], h.pos[1], prop);  // propagate-tor-test_hip.cu:842-845
     }
-    float c = Lane<EXACT>::update(prop, h);
+    float c = Lane<EXACT>::update(prop, h, r);
     if (opts) apply_options<EXACT>(opts, prop, q, k, kfact);
     if (SEM == P2R_REFERENCE) {
       // Only the last layer's result is returned in reference semantics; the
@@ -240,8 +241,8 @@ __device__ __forceinline__ void ragged_slot(const float* __restrict__ trk, const
       src = cur;
     }
     Trk prop;
-    Lane<EXACT>::propagate(src, k, h.pos[0], h.pos[1], prop);
-    float c = Lane<EXACT>::update(prop, h);
+    const float r = Lane<EXACT>::propagate(src.par, src.cov, k, h.pos[0], h.pos[1], prop);
+    float c = Lane<EXACT>::update(prop, h, r);
     if (opts) apply_options<EXACT>(opts, prop, q, k, kfact);
     if (SEM == P2R_REFERENCE) {
       opaque(prop);
@@ -387,8 +388,8 @@ __global__ __launch_bounds__(kThreads) void fwd_ragged_layer_kernel(const float*
         src = cur;
       }
       Trk prop;
-      Lane<EXACT>::propagate(src, k, h.pos[0], h.pos[1], prop);
-      float c = Lane<EXACT>::update(prop, h);
+      const float r = Lane<EXACT>::propagate(src.par, src.cov, k, h.pos[0], h.pos[1], prop);
+      float c = Lane<EXACT>::update(prop, h, r);
       if (opts) apply_options<EXACT>(opts, prop, q, k, kfact);
       if (SEM == P2R_REFERENCE) {
         opaque(prop);
@@ -558,8 +559,8 @@ __global__ __launch_bounds__(64 * kPsWaves) void fwd_ragged_stream_kernel(const 
       float k = (float)q * kfact;
       if (SEM == P2R_REFERENCE) opaque(src);
       Trk prop;
-      Lane<EXACT>::propagate(src, k, h.pos[0], h.pos[1], prop);
-      float cc = Lane<EXACT>::update(prop, h);
+      const float r = Lane<EXACT>::propagate(src.par, src.cov, k, h.pos[0], h.pos[1], prop);
+      float cc = Lane<EXACT>::update(prop, h, r);
       if (opts) apply_options<EXACT>(opts, prop, q, k, kfact);
       if (SEM == P2R_REFERENCE) {
         opaque(prop);
@@ -640,8 +641,7 @@ template <class R, bool EXACT> struct MathOf;
 template <> struct MathOf<float, true> {
   using T = exact::Trk; using H = exact::Hit;
   static __device__ __forceinline__ float fwd(const T& in, float k, const H& h, T& out) {
-    exact::propagate_to_r(in, k, h.pos[0], h.pos[1], out);
-    return exact::kalman_update(out, h);
+    return exact::kalman_update_r(out, h, exact::propagate_to_r(in, k, h.pos[0], h.pos[1], out));
   }
   static __device__ __forceinline__ void adj(const T& in, float k, const H& h, T& bar, float& kb, float hb[3]) {
     exact::layer_adjoint(in, k, h, bar, kb, hb);
@@ -650,8 +650,7 @@ template <> struct MathOf<float, true> {
 template <> struct MathOf<float, false> {
   using T = fast::Trk; using H = fast::Hit;
   static __device__ __forceinline__ float fwd(const T& in, float k, const H& h, T& out) {
-    fast::propagate_to_r(in, k, h.pos[0], h.pos[1], out);
-    return fast::kalman_update(out, h);
+    return fast::kalman_update_r(out, h, fast::propagate_to_r(in, k, h.pos[0], h.pos[1], out));
   }
   static __device__ __forceinline__ void adj(const T& in, float k, const H& h, T& bar, float& kb, float hb[3]) {
     fast::layer_adjoint(in, k, h, bar, kb, hb);
@@ -660,8 +659,7 @@ template <> struct MathOf<float, false> {
 template <bool EXACT> struct MathOf<double, EXACT> {
   using T = dbl::Trk; using H = dbl::Hit;
   static __device__ __forceinline__ double fwd(const T& in, double k, const H& h, T& out) {
-    dbl::propagate_to_r(in, k, h.pos[0], h.pos[1], out);
-    return dbl::kalman_update(out, h);
+    return dbl::kalman_update_r(out, h, dbl::propagate_to_r(in, k, h.pos[0], h.pos[1], out));
   }
   static __device__ __forceinline__ void adj(const T& in, double k, const H& h, T& bar, double& kb, double hb[3]) {
     dbl::layer_adjoint(in, k, h, bar, kb, hb);
@@ -1047,7 +1045,7 @@ __global__ __launch_bounds__(kThreads) void propagate_blocks_kernel(const float*
   for (int f = 0; f < 21; ++f) in.cov[f] = inErr[to + (size_t)f * bs];
   const float k = (float)inChg[to] * kfact;
   Trk o;
-  Lane<true>::propagate(in, k, msP[ho], msP[ho + bs], o);
+  Lane<true>::propagate(in.par, in.cov, k, msP[ho], msP[ho + bs], o);
 #pragma unroll
   for (int f = 0; f < 6; ++f) outPar[to + (size_t)f * bs] = o.par[f];
 #pragma unroll

@@ -33,6 +33,8 @@ __device__ __forceinline__ void opaque(double& v) { asm volatile("" : "+v"(v)); 
 // No instruction is scheduled across this point (code size 0): separates phases whose values should not
 // be live at the same time.
 __device__ __forceinline__ void phase_boundary() { __builtin_amdgcn_sched_barrier(0); }
+// True in every active lane of the wavefront when `v` holds in one of them.
+__device__ __forceinline__ bool any_lane(bool v) { return __ballot(v) != 0; }
 __device__ __forceinline__ void opaque(Trk& t) {
 #pragma unroll
   for (int i = 0; i < 6; ++i) opaque(t.par[i]);
@@ -57,6 +59,22 @@ template <class A, class B> __device__ __forceinline__ void convert(const HitT<A
 // FP64 instance's division and square root and in the fast instance's FP64 reciprocal.
 __device__ __forceinline__ double rcp_est(double x) { return __builtin_amdgcn_rcp(x); }
 __device__ __forceinline__ double rsq_est(double x) { return __builtin_amdgcn_rsq(x); }
+
+// Hardware estimates at raised wave priority, for code that runs with several wavefronts per SIMD.  Such a SIMD
+// starts an FP32 instruction every 2.1 cycles, from two wavefronts in turn, but one plain quarter-rate instruction
+// (v_rcp, v_rsq, v_sqrt), v_div_fmas or v_readfirstlane takes it out of that rhythm for tens of instructions: a
+// stream with one v_rcp_f32 in 25 issues at 4.1 cycles per instruction, with s_setprio around the v_rcp at 2.5 (4
+// wavefronts per SIMD).  The s_setprio after it is also the wait state that its first reader needs.
+#define P2R_PRIO(name, T, op)                                                                       \
+  __device__ __forceinline__ T name(T x) {                                                          \
+    T y;                                                                                            \
+    asm("s_setprio 1\n\t" op " %0, %1\n\ts_setprio 0" : "=v"(y) : "v"(x));                          \
+    return y;                                                                                       \
+  }
+P2R_PRIO(rcp_prio, float, "v_rcp_f32_e32")
+P2R_PRIO(rsq_prio, float, "v_rsq_f32_e32")
+P2R_PRIO(rcp_prio, double, "v_rcp_f64_e32")
+#undef P2R_PRIO
 
 // Instances of the per-lane math (see p2r_lane_math.inc) and of its adjoint
 // (p2r_adjoint.inc).
@@ -104,30 +122,29 @@ using Jac = JacT<real>;
 #undef P2R_DOUBLE_EST
 }  // namespace dbl
 
-// Compile-time selection of the instance.
+// Compile-time selection of the instance.  propagate returns the hit's radius, for the update of the same layer.
 template <bool EXACT> struct Lane;
 template <> struct Lane<true> {
-  static __device__ __forceinline__ void propagate(const Trk& in, float k, float hx, float hy, Trk& out) {
-    exact::propagate_to_r(in, k, hx, hy, out);
-  }
   template <class PC>
-  static __device__ __forceinline__ void propagate(const float (&par)[6], const PC& P, float k, float hx, float hy,
-                                                   Trk& out) {
-    exact::propagate_to_r_c(par, P, k, hx, hy, out);
+  static __device__ __forceinline__ float propagate(const float (&par)[6], const PC& P, float k, float hx, float hy,
+                                                    Trk& out) {
+    return exact::propagate_to_r_c(par, P, k, hx, hy, out);
+  }
+  static __device__ __forceinline__ float update(Trk& t, const Hit& h, float r) {
+    return exact::kalman_update_r(t, h, r);
   }
   static __device__ __forceinline__ float update(Trk& t, const Hit& h) { return exact::kalman_update(t, h); }
   static __device__ __forceinline__ float wrap_phi(float phi) { return exact::m_wrap_phi(phi); }
 };
 template <> struct Lane<false> {
-  static __device__ __forceinline__ void propagate(const Trk& in, float k, float hx, float hy, Trk& out) {
-    fast::propagate_to_r(in, k, hx, hy, out);
-  }
   template <class PC>
-  static __device__ __forceinline__ void propagate(const float (&par)[6], const PC& P, float k, float hx, float hy,
-                                                   Trk& out) {
-    fast::propagate_to_r_c(par, P, k, hx, hy, out);
+  static __device__ __forceinline__ float propagate(const float (&par)[6], const PC& P, float k, float hx, float hy,
+                                                    Trk& out) {
+    return fast::propagate_to_r_c(par, P, k, hx, hy, out);
   }
-  static __device__ __forceinline__ float update(Trk& t, const Hit& h) { return fast::kalman_update(t, h); }
+  static __device__ __forceinline__ float update(Trk& t, const Hit& h, float r) {
+    return fast::kalman_update_r(t, h, r);
+  }
   static __device__ __forceinline__ float wrap_phi(float phi) { return fast::m_wrap_phi(phi); }
 };
 
