@@ -195,6 +195,81 @@ __global__ __launch_bounds__(kThreads, MINW) void fwd_uniform_kernel(const float
 }
 
 
+// Reference semantics for batches too small to fill the chip with one wavefront per 64 tracks: every layer starts
+// from the input track, so the layers of a tile are dealt to wavefronts of their own.  Workgroup (x, y) takes
+// tile x's layers [y, y + 1) * blockDim.x / 64 * per_wave, wavefront w of it per_wave of them; the tile's input
+// covariance waits in LDS for all of them, and the last layer's wavefront writes the track, after the barrier
+// that follows the workgroup's reads of it.  The chi2 sum over a track's layers is taken in layer order from LDS,
+// so it needs all the layers in one workgroup (gridDim.y == 1), as does trk_out over trk_in.
+// Bound by the latency of a wavefront's layers: with one wavefront per tile, an event's 150 took 50.5 us (exact, 9600
+// tracks x 20 layers) on 150 of the 1024 SIMDs, a layer after the other at an instruction per 4.3 cycles; with the
+// layers dealt out it takes 10.9, most of which is the launch.
+constexpr int kTileTracks = 64;
+template <bool CHI2, bool EXACT>
+__global__ __launch_bounds__(1024) void fwd_layers_kernel(const float* trk, const float* __restrict__ hits, float* out,
+                                                          float* __restrict__ chi2, uint32_t ntrk, uint32_t bs,
+                                                          int nlayer, float kfact, int per_wave, int opts) {
+  extern __shared__ float lds[];  // [64][21] covariance, then [nlayer][64] chi2 when it is summed
+  const bool per_layer = opts & P2R_OPT_CHI2_PER_LAYER;
+  const uint32_t lane_id = threadIdx.x & 63u;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), nwaves = blockDim.x >> 6;
+  const uint32_t g = blockIdx.x * kTileTracks + lane_id;
+  const bool active = g < ntrk;
+  const uint32_t gg = active ? g : ntrk - 1u;
+  const uint32_t blk = gg / bs, lane = gg - blk * bs;
+  const float* tb = trk + (size_t)blk * 28 * bs + lane;
+  float* cov_lds = lds;
+  float* c_lds = lds + kTileTracks * 21;
+  float in_par[6];
+#pragma unroll
+  for (int f = 0; f < 6; ++f) in_par[f] = tb[(size_t)f * bs];
+  for (int f = wave; f < 21; f += nwaves) cov_lds[lane_id * 21u + f] = tb[(size_t)(6 + f) * bs];
+  const int q_in = reinterpret_cast<const int*>(tb)[(size_t)27 * bs];
+  __syncthreads();
+  if (active) {
+    const WaveHits wh(hits, g, ntrk, bs, nlayer, blk, lane);
+    const int first = (int)(blockIdx.y * nwaves + wave) * per_wave;
+    const int last = min(first + per_wave, nlayer);
+    Trk cur;
+    int q = q_in;
+    for (int l = first; l < last; ++l) {
+      Hit h;
+      wh.load(l, h);
+      // every layer recomputes and rereads the input, as in fwd_uniform_kernel
+#pragma unroll
+      for (int f = 0; f < 6; ++f) opaque(in_par[f]);
+      uint32_t col = lane_id;
+      asm volatile("" : "+v"(col));
+      q = q_in;
+      float k = (float)q * kfact;
+      Trk prop;
+      const float r = Lane<EXACT>::propagate(in_par, LdsCov{cov_lds + col * 21u}, k, h.pos[0], h.pos[1], prop);
+      float c = Lane<EXACT>::update(prop, h, r);
+      if (opts) apply_options<EXACT>(opts, prop, q, k, kfact);
+      opaque(prop);
+      opaque(c);
+      if (CHI2) {
+        if (per_layer) chi2[(size_t)l * ntrk + g] = c;
+        else c_lds[l * kTileTracks + lane_id] = c;
+      }
+      cur = prop;
+    }
+    if (first < nlayer && last == nlayer) {
+      float* ob = out + (size_t)blk * 28 * bs + lane;
+      store_trk(ob, bs, cur);
+      reinterpret_cast<int*>(ob)[(size_t)27 * bs] = q;
+    }
+  }
+  if (CHI2) {
+    if (per_layer) return;
+    __syncthreads();
+    if (wave != 0 || !active) return;
+    float c2 = 0.f;
+    for (int l = 0; l < nlayer; ++l) c2 += c_lds[l * kTileTracks + lane_id];
+    chi2[g] = c2;
+  }
+}
+
 // ---------------------------------------------------------------------------
 // Uneven batch: persistent workgroups walk tiles of kRagThreads*ROUNDS
 // consecutive slots.  Within a tile, slots are ordered by hit count (stable,
@@ -1120,12 +1195,48 @@ void launch_uniform_p(bool exact, int waves, dim3 grid, dim3 block, hipStream_t 
   if (exact) launch_uniform_e<SEM, CHI2, true>(waves, grid, block, st, a, in, l0, l1, acc);
   else launch_uniform_e<SEM, CHI2, false>(waves, grid, block, st, a, in, l0, l1, acc);
 }
+// How a small batch's layers are dealt to wavefronts (fwd_layers_kernel), in reference semantics: per_wave layers to
+// each of `waves` wavefronts of a workgroup, `groups` workgroups per tile of 64 tracks; waves == 0: not at all.
+struct LayerSplit {
+  int waves = 0, groups = 0, per_wave = 0;
+};
+LayerSplit split_layers(int num_cus, uint64_t ntrk, int nlayer, bool one_group) {
+  // The line: from 2 wavefronts per SIMD on (4 SIMDs a CU) fwd_uniform_kernel fills the issue slots by itself.
+  // Exact x 20 layers, split against not, us: 512 tiles 18.7 / 51.6, 1024 31.2 / 52.9, 1500 53.0 / 58.3, 2048 60.7 /
+  // 60.8; beyond that a static division only adds imbalance.
+  const uint64_t tiles = (ntrk + kTileTracks - 1) / kTileTracks, simds = (uint64_t)num_cus * 4;
+  LayerSplit s;
+  if (nlayer < 2 || tiles > 2 * simds) return s;
+  // about 4 wavefronts per SIMD in all
+  const int m = std::max<int>(1, (int)((tiles * nlayer + 4 * simds - 1) / (4 * simds)));
+  const int want = (nlayer + m - 1) / m;  // wavefronts per tile
+  if (want < 2) return s;
+  s.waves = std::min(want, one_group ? 16 : 4);
+  s.per_wave = one_group ? (nlayer + s.waves - 1) / s.waves : m;
+  s.groups = one_group ? 1 : (nlayer + s.waves * m - 1) / (s.waves * m);
+  return s;
+}
 // The whole forward: one launch over all layers, or launches of `per_launch`
 // layers (the state passes through trk_out between launches; in reference
 // semantics every launch restarts from trk_in, as every layer does, and only
 // the last launch writes trk_out).
-void launch_uniform(int sem, bool exact, int threads, int per_launch, int waves, hipStream_t st,
+void launch_uniform(int num_cus, int sem, bool exact, int threads, int per_launch, int waves, hipStream_t st,
                     const UniformLaunch& a) {
+  if (sem == P2R_REFERENCE && (per_launch <= 0 || per_launch >= a.nlayer)) {
+    const bool summed = a.chi2 && !(a.opts & P2R_OPT_CHI2_PER_LAYER);
+    const bool in_place = overlaps(a.T, (size_t)a.n * 112, a.O, (size_t)a.n * 112);
+    const LayerSplit s = split_layers(num_cus, a.n, a.nlayer, summed || in_place);
+    if (s.waves) {
+      const dim3 grid((unsigned)((a.n + kTileTracks - 1) / kTileTracks), (unsigned)s.groups), block(64 * s.waves);
+      const size_t lds = sizeof(float) * kTileTracks * (21 + (summed ? a.nlayer : 0));
+      auto go = [&](auto kernel) {
+        kernel<<<grid, block, lds, st>>>(a.T, a.H, a.O, a.chi2, a.n, a.bs, a.nlayer, a.kf, s.per_wave, a.opts);
+      };
+      if (a.chi2) exact ? go(fwd_layers_kernel<true, true>) : go(fwd_layers_kernel<true, false>);
+      else exact ? go(fwd_layers_kernel<false, true>) : go(fwd_layers_kernel<false, false>);
+      return;
+    }
+  }
   const dim3 grid(grid_for_n(a.n, threads)), block(threads);
   const int step = (per_launch > 0 && per_launch < a.nlayer) ? per_launch : a.nlayer;
   for (int l0 = 0; l0 < a.nlayer; l0 += step) {
@@ -1477,7 +1588,7 @@ int p2r_forward(p2r_ctx* c, const void* trk_in, const void* hits, void* trk_out,
   DeviceGuard g(c->device);
   const UniformLaunch a{static_cast<const float*>(trk_in), static_cast<const float*>(hits), static_cast<float*>(trk_out),
                         chi2, (uint32_t)ntrk, (uint32_t)s->bsize, s->nlayer, p.kfact / p.b_scale, p.options};
-  launch_uniform(semantics, p.precision == P2R_EXACT, c->tune.fwd_threads, c->tune.fwd_layers_per_launch,
+  launch_uniform(c->num_cus, semantics, p.precision == P2R_EXACT, c->tune.fwd_threads, c->tune.fwd_layers_per_launch,
                  c->tune.fwd_waves, static_cast<hipStream_t>(stream), a);
   return c->check_launch("p2r_forward");
 }
@@ -1533,7 +1644,7 @@ int p2r_forward_streamed(p2r_ctx* c, const void* host_trk_in, const void* host_h
     const UniformLaunch a{reinterpret_cast<const float*>(dt), reinterpret_cast<const float*>(dh),
                           reinterpret_cast<float*>(dout), nullptr, (uint32_t)(nb * bs), (uint32_t)bs, s->nlayer,
                           p.kfact / p.b_scale, p.options};
-    launch_uniform(semantics, p.precision == P2R_EXACT, c->tune.fwd_threads, c->tune.fwd_layers_per_launch,
+    launch_uniform(c->num_cus, semantics, p.precision == P2R_EXACT, c->tune.fwd_threads, c->tune.fwd_layers_per_launch,
                    c->tune.fwd_waves, st, a);
     const int rc = c->check_launch("p2r_forward_streamed");
     if (rc != P2R_OK) {
