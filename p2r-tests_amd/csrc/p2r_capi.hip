@@ -725,7 +725,7 @@ template <> struct MathOf<float, true> {
 template <> struct MathOf<float, false> {
   using T = fast::Trk; using H = fast::Hit;
   static __device__ __forceinline__ float fwd(const T& in, float k, const H& h, T& out) {
-    return fast::kalman_update_r(out, h, fast::propagate_to_r(in, k, h.pos[0], h.pos[1], out));
+    return fast::fast_update(out, h, fast::fast_propagate(in.par, in.cov, k, h.pos[0], h.pos[1], out));
   }
   static __device__ __forceinline__ void adj(const T& in, float k, const H& h, T& bar, float& kb, float hb[3]) {
     fast::layer_adjoint(in, k, h, bar, kb, hb);

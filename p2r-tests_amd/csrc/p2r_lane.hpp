@@ -14,6 +14,7 @@
 // structural zeros and ones, including row 3 (a unit row) which the reference
 // multiplies out generically (tbb.cpp:322-327, 357-360); for finite inputs the
 // result is identical.
+// The fast instance regroups the layer (p2r_fast_layer.inc).
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -101,6 +102,7 @@ using Jac = JacT<real>;
 #define P2R_EXACT 0
 #define P2R_DOUBLE 0
 #include "p2r_lane_math.inc"
+#include "p2r_fast_layer.inc"
 #include "p2r_adjoint.inc"
 #undef P2R_EXACT
 #undef P2R_DOUBLE
@@ -122,7 +124,8 @@ using Jac = JacT<real>;
 #undef P2R_DOUBLE_EST
 }  // namespace dbl
 
-// Compile-time selection of the instance.  propagate returns the hit's radius, for the update of the same layer.
+// Compile-time selection of the instance.  propagate returns what the update of the same layer needs of it: the
+// hit's radius (exact), its reciprocal (fast).
 template <bool EXACT> struct Lane;
 template <> struct Lane<true> {
   template <class PC>
@@ -140,10 +143,10 @@ template <> struct Lane<false> {
   template <class PC>
   static __device__ __forceinline__ float propagate(const float (&par)[6], const PC& P, float k, float hx, float hy,
                                                     Trk& out) {
-    return fast::propagate_to_r_c(par, P, k, hx, hy, out);
+    return fast::fast_propagate(par, P, k, hx, hy, out);
   }
   static __device__ __forceinline__ float update(Trk& t, const Hit& h, float r) {
-    return fast::kalman_update_r(t, h, r);
+    return fast::fast_update(t, h, r);
   }
   static __device__ __forceinline__ float wrap_phi(float phi) { return fast::m_wrap_phi(phi); }
 };
