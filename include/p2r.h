@@ -180,7 +180,8 @@ typedef enum p2r_grad_precision { P2R_GRAD_F32 = 0, P2R_GRAD_MIXED = 1, P2R_GRAD
  * ntrk states of 4 bytes (P2R_GRAD_F32) or 8 bytes, plus (stride - 2) * 27 *
  * ntrk values for the recomputed layer inputs of a segment where they do not
  * fit in LDS (stride 8, and stride 4 with F64), of 4 bytes (F32, MIXED) or 8
- * (F64).  The context holds one
+ * (F64).  A batch whose states of every layer fit 48 MiB of workspace keeps
+ * them all, whatever the stride.  The context holds one
  * workspace: adjoint calls on one context must not overlap in time (issue
  * them on one stream, or synchronize between streams or threads).
  * trk_out must not overlap trk_in (the reverse sweep rereads the input

@@ -1368,6 +1368,13 @@ int resolve_scratch(int device, void** out) {
   return P2R_OK;
 }
 
+// A batch whose states of every layer fit this much workspace keeps them all, whatever the checkpoint stride: it is
+// bound by the latency of its few wavefronts, and recomputing a segment's states from its checkpoint only lengthens
+// them.  9600 tracks x 20 layers (38 MB of FP64 states) at stride 4, us: F64 202 -> 173, 2048 tracks MIXED
+// through autograd 192 -> 184.  Larger batches hide the recompute and would pay for the states' traffic (960 000 tracks
+// MIXED: 2.25 ms at stride 4, 2.45 at stride 1).
+constexpr size_t kSmallAdjointBytes = 48u << 20;
+
 // Validated arguments and workspace layout of one adjoint call.
 struct AdjointPlan {
   uint32_t n = 0, bs = 0;
@@ -1407,20 +1414,24 @@ int adjoint_plan(p2r_ctx* c, const void* trk_in, const void* hits, const void* t
   pl.bs = (uint32_t)s->bsize;
   pl.nlayer = s->nlayer;
   pl.nglob = 4 * s->nlayer + 1;
-  pl.cs = cs;
   pl.grad_precision = grad_precision;
   pl.p = p;
   if (ntrk == 0) return P2R_OK;
   pl.grid = grid_for_n(ntrk, kAdjThreads);
-  const size_t sz = grad_precision == P2R_GRAD_F32 ? sizeof(float) : sizeof(double);
-  const size_t nck = (size_t)((pl.nlayer + cs - 1) / cs - 1);
-  pl.ck_bytes = std::max<size_t>(nck, 1) * 27 * ntrk * sz;
-  pl.c2_bytes = ntrk * sz;
-  pl.part_bytes = global ? (size_t)pl.grid * pl.nglob * sizeof(double) : 0;
-  pl.seg_bytes = seg_global_bytes(grad_precision, cs, ntrk);
-  pl.bar_bytes = grad_precision == P2R_GRAD_MIXED ? (size_t)28 * sizeof(float) * ntrk : 0;
-  pl.ws_bytes = ck_bytes_aligned(pl.ck_bytes) + ck_bytes_aligned(pl.c2_bytes) + ck_bytes_aligned(pl.part_bytes) +
-                ck_bytes_aligned(pl.seg_bytes) + pl.bar_bytes + 256;
+  auto lay_out = [&](int stride) {
+    pl.cs = stride;
+    const size_t sz = grad_precision == P2R_GRAD_F32 ? sizeof(float) : sizeof(double);
+    const size_t nck = (size_t)((pl.nlayer + stride - 1) / stride - 1);
+    pl.ck_bytes = std::max<size_t>(nck, 1) * 27 * ntrk * sz;
+    pl.c2_bytes = ntrk * sz;
+    pl.part_bytes = global ? (size_t)pl.grid * pl.nglob * sizeof(double) : 0;
+    pl.seg_bytes = seg_global_bytes(grad_precision, stride, ntrk);
+    pl.bar_bytes = grad_precision == P2R_GRAD_MIXED ? (size_t)28 * sizeof(float) * ntrk : 0;
+    pl.ws_bytes = ck_bytes_aligned(pl.ck_bytes) + ck_bytes_aligned(pl.c2_bytes) + ck_bytes_aligned(pl.part_bytes) +
+                  ck_bytes_aligned(pl.seg_bytes) + pl.bar_bytes + 256;
+  };
+  lay_out(1);
+  if (pl.ws_bytes > kSmallAdjointBytes) lay_out(cs);
   pl.lds = global ? (size_t)(kAdjThreads / 64) * pl.nglob * sizeof(double) : 0;
   return P2R_OK;
 }
