@@ -79,3 +79,30 @@ def test_exact_propagation_at_the_ends_of_kfact(orc, ctx, kfact):
             assert same.all()
     finally:
         orc.lib.orc_set_trig_mode(0)
+
+
+# angles (FP32 bits) whose sine or cosine lies within 250 ulps of FP64 of the midpoint between two floats
+UNSURE = [0xc0259f7c, 0x40096e02, 0xbfe3343a, 0xc04549a0, 0xbfe9c645, 0x3e659fc6, 0x3cb0bc91, 0x4010a4bf, 0x3ffedd26,
+          0x3fadffc7, 0xbe5c11ed]
+# the ends of the range of the kernels' own sine and cosine, and around it; multiples of pi/2
+ANGLES = [2.0 ** -24, np.nextafter(np.float32(2.0 ** -24), np.float32(0)), -(2.0 ** -30), 0.0, -0.0, 1e-40, 4096.0,
+          np.nextafter(np.float32(4096), np.float32(5000)), -4095.9, 1e5, 3e38, np.inf, np.nan,
+          *(k * np.pi / 2 for k in (-2607, -5, -2, -1, 1, 2, 3, 4, 101, 2607)), np.pi / 4, -3 * np.pi / 4, 2.356]
+
+
+@pytest.mark.parametrize("field", [4, 5])
+@pytest.mark.parametrize("semantics", ["reference", "chained"])
+def test_exact_sine_and_cosine_words(orc, ctx, semantics, field):
+    """phi (4) and theta (5) at the ends of their range, at multiples of pi/2 and where the FP32 rounding of a sine or
+    cosine is in doubt, one per wavefront and all in a few wavefronts."""
+    from test_gpu_parity import check_exact
+    import p2r_amd
+    angles = np.concatenate([np.array(UNSURE, np.uint32).view(np.float32), np.array(ANGLES, np.float32)])
+    for spread in (64, 1):
+        n = 32 * (-(-len(angles) * spread // 32))
+        shape = Shape(1, n, 2, 32)
+        trk, hits = p2r_amd.gen_uniform(shape)
+        t = trk.reshape(shape.nblk, 28, 32)
+        for i, a in enumerate(angles):
+            t[i * spread // 32, field, i * spread % 32] = a
+        check_exact(orc, ctx, trk, hits, shape, semantics, f"angles field {field} spread {spread}")
