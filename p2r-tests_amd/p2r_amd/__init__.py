@@ -25,13 +25,31 @@ def _ptr(t):
         return None
     if isinstance(t, np.ndarray):
         return t.ctypes.data_as(C.c_void_p)
-    return C.c_void_p(t.data_ptr())
+    return t.data_ptr()  # every pointer parameter is a c_void_p
+
+
+# torch, imported with the first call that needs it: (module, {kind: dtype}, raw handle of a device's current stream)
+_torch_cache = None
+
+
+def _torch():
+    global _torch_cache
+    if _torch_cache is None:
+        import torch
+        _torch_cache = (torch, {k: getattr(torch, v) for k, v in _TORCH_DTYPES.items()},
+                        getattr(torch._C, "_cuda_getCurrentRawStream", None))
+    return _torch_cache
 
 
 def _stream(stream):
-    import torch
-    s = torch.cuda.current_stream() if stream is None else stream
-    return C.c_void_p(s.cuda_stream)
+    """A stream's handle, by default the current device's current stream (a Stream object for it takes 2.6 us to make,
+    the handle 0.3)."""
+    if stream is not None:
+        return stream.cuda_stream
+    torch, _, raw = _torch()
+    if raw is not None and torch.cuda.is_initialized():
+        return raw(torch.cuda.current_device())
+    return torch.cuda.current_stream().cuda_stream
 
 
 # ---- buffer checks --------------------------------------------------------------------------------------
@@ -43,21 +61,21 @@ def _stream(stream):
 _TORCH_DTYPES = {"f32": "float32", "i32": "int32", "f64": "float64"}
 
 
-def _check_dev(t, n, kind, device, name):
+def _check_dev(t, n, kind, device, name, call="buffer"):
     if t is None or n <= 0:
         return
-    import torch
+    torch, dtypes, _ = _torch()
     if not isinstance(t, torch.Tensor) or not t.is_cuda:
-        raise TypeError(f"{name}: expected a CUDA tensor, got {type(t).__name__}"
+        raise TypeError(f"{call}: {name}: expected a CUDA tensor, got {type(t).__name__}"
                         + ("" if not isinstance(t, torch.Tensor) else f" on {t.device}"))
-    if t.device.index != device:
-        raise ValueError(f"{name}: tensor on {t.device}, context on cuda:{device}")
-    if t.dtype != getattr(torch, _TORCH_DTYPES[kind]):
-        raise TypeError(f"{name}: dtype {t.dtype}, expected torch.{_TORCH_DTYPES[kind]}")
+    if t.get_device() != device:
+        raise ValueError(f"{call}: {name}: tensor on {t.device}, context on cuda:{device}")
+    if t.dtype != dtypes[kind]:
+        raise TypeError(f"{call}: {name}: dtype {t.dtype}, expected torch.{_TORCH_DTYPES[kind]}")
     if not t.is_contiguous():
-        raise ValueError(f"{name}: tensor is not contiguous")
+        raise ValueError(f"{call}: {name}: tensor is not contiguous")
     if t.numel() < n:
-        raise ValueError(f"{name}: {t.numel()} elements, the shape needs {n}")
+        raise ValueError(f"{call}: {name}: {t.numel()} elements, the shape needs {n}")
 
 
 def _check_host(t, n, name):
@@ -165,7 +183,7 @@ class Context:
         n = sh.nevts * sh.ntrks
         for t, m, name in ((trk, 28 * n, "trk"), (hits, 9 * n * sh.nlayer, "hits"), (out, 28 * n, "out"),
                            (chi2, n * (sh.nlayer if p.options & P2R_OPT_CHI2_PER_LAYER else 1), "chi2")):
-            _check_dev(t, m, "f32", self.device, f"{what}: {name}")
+            _check_dev(t, m, "f32", self.device, name, what)
 
     def _check_ragged(self, trk, hits, out, offs, mask, nlayer, bsize, p, chi2, what):
         if not (_ragged_ok(offs, nlayer, bsize) and _params_ok(p)):
@@ -173,8 +191,8 @@ class Context:
         nslot = int(offs[-1]) * bsize
         for t, m, name in ((trk, 28 * nslot, "trk"), (hits, 9 * nslot * nlayer, "hits"), (out, 28 * nslot, "out"),
                            (chi2, nslot * (nlayer if p.options & P2R_OPT_CHI2_PER_LAYER else 1), "chi2")):
-            _check_dev(t, m, "f32", self.device, f"{what}: {name}")
-        _check_dev(mask, nslot, "i32", self.device, f"{what}: layer_mask")
+            _check_dev(t, m, "f32", self.device, name, what)
+        _check_dev(mask, nslot, "i32", self.device, "layer_mask", what)
 
     def _check_adjoint(self, trk, hits, out, sh, p, gp, cs, chi2, grad_par, grad_hits, grad_kfact, grad_global,
                        what):
@@ -185,8 +203,8 @@ class Context:
         for t, m, name in ((trk, 28 * n, "trk"), (hits, 9 * n * L, "hits"), (out, 28 * n, "out"), (chi2, n, "chi2"),
                            (grad_par, 6 * n, "grad_par"), (grad_hits, 3 * n * L, "grad_hits"),
                            (grad_kfact, n, "grad_kfact")):
-            _check_dev(t, m, "f32", self.device, f"{what}: {name}")
-        _check_dev(grad_global, 4 * L + 1, "f64", self.device, f"{what}: grad_global")
+            _check_dev(t, m, "f32", self.device, name, what)
+        _check_dev(grad_global, 4 * L + 1, "f64", self.device, "grad_global", what)
 
     def forward(self, trk, hits, out, shape, semantics="reference", params=None, chi2=None, stream=None,
                 precision=None):
@@ -357,8 +375,8 @@ class Context:
         """Matriplex width conversion on the device (MPTRK: nsub=1, words=28; MPHIT: nsub=nlayer, words=9)."""
         total = int(nevts) * int(ntrks) * int(nsub) * int(words)
         if total > 0 and nsub >= 1 and words >= 1:
-            _check_dev(src, total, "f32", self.device, "p2r_repack: src")
-            _check_dev(dst, total, "f32", self.device, "p2r_repack: dst")
+            _check_dev(src, total, "f32", self.device, "src", "p2r_repack")
+            _check_dev(dst, total, "f32", self.device, "dst", "p2r_repack")
         self._check(lib().p2r_repack(self._h, _ptr(src), int(src_bsize), _ptr(dst), int(dst_bsize), int(nevts),
                                      int(ntrks), int(nsub), int(words), _stream(stream)), "p2r_repack")
 
