@@ -809,7 +809,7 @@ __global__ __launch_bounds__(kAdjThreads, MINW) void adjoint_fwd_kernel(
 #pragma unroll
       for (int f = 0; f < 21; ++f) cp[(size_t)(6 + f) * ntrk] = cur.cov[f];
     }
-    HitT<RS> h;  // loaded as the layer starts (no prefetch: 127 instead of 153 VGPRs in FP32, 4 waves)
+    HitT<RS> h;  // loaded as the layer starts (no prefetch: 125 VGPRs in exact FP32, 4 waves)
     load_hit_as(hb + l * hstride, bs, h);
     TrkT<RS> nxt;
     c2 += MS::fwd(cur, (RS)k, h, nxt);
@@ -1181,9 +1181,9 @@ void launch_uniform_w(dim3 grid, dim3 block, hipStream_t st, const UniformLaunch
 template <int SEM, bool CHI2, bool EXACT>
 void launch_uniform_e(int waves, dim3 grid, dim3 block, hipStream_t st, const UniformLaunch& a, const float* in,
                       int l0, int l1, bool acc) {
-  // 0 = the library's choice: the 3-wave budget for the exact instance, 4 waves for the fast one.  The
-  // current kernels fit 5 or more waves per SIMD at the compiler's own allocation, and the three budgets
-  // compile to the same instructions; the choice stays for the autotuner.
+  // 0 = the library's choice: the 3-wave budget for the exact instance, 4 waves for the fast one.  At every
+  // budget the exact kernels fit 4 waves per SIMD (97-127 VGPRs) and the fast ones 5 or 6 (73-92), without
+  // spills, and run alike within noise; the choice stays for the autotuner.
   if (waves == 0) waves = EXACT ? 3 : 4;
   if (waves == 3) launch_uniform_w<SEM, CHI2, EXACT, 3>(grid, block, st, a, in, l0, l1, acc);
   else if (waves == 4) launch_uniform_w<SEM, CHI2, EXACT, 4>(grid, block, st, a, in, l0, l1, acc);
