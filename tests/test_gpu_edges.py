@@ -68,6 +68,13 @@ def test_exact_partial_wavefronts(orc, ctx, nevts, ntrks, bsize):
         assert _same(gpu, cpu) and _same(c2g, c2c), sem
 
 
+def _words(ctx, trk, hits, shape, semantics, precision):
+    dt, dh = torch.from_numpy(trk).cuda(), torch.from_numpy(hits).cuda()
+    do = torch.empty_like(dt)
+    ctx.forward(dt, dh, do, shape, semantics, precision=precision)
+    return do.cpu().numpy().view(np.uint32).reshape(-1, 28, shape.bsize).copy()
+
+
 def test_exact_widest_matriplex(orc, ctx):
     import p2r_amd
     shape = Shape(1, 2048, 20, 1024)
@@ -77,6 +84,24 @@ def test_exact_widest_matriplex(orc, ctx):
         cpu, c2c = orc.run_f32(trk, hits, shape.nblk, 20, 1024, semantics=0 if sem == "reference" else 1,
                                chi2=True, cr_trig=True)
         assert _same(gpu, cpu) and _same(c2g, c2c)
+
+
+@pytest.mark.parametrize("semantics", ["reference", "chained"])
+@pytest.mark.parametrize("precision", ["exact", "fast"])
+@pytest.mark.parametrize("ntrks", [64, 131136])
+def test_hit_on_the_z_axis_has_no_finite_result(ctx, semantics, precision, ntrks):
+    """A hit at x = y = 0 (radius 0, no tangent plane) gives its track NaN in every word in both arithmetics, and its
+    wavefront's other tracks what they are without it; below and above the line of the layer split."""
+    import p2r_amd
+    shape = Shape(1, ntrks, 2, 32)
+    trk, hits = p2r_amd.gen_uniform(shape)
+    h = hits.reshape(-1, 2, 9, 32)
+    clean = _words(ctx, trk, hits, shape, semantics, precision)
+    h[1, 1, :2, 7] = 0.0
+    got = _words(ctx, trk, hits, shape, semantics, precision)
+    assert np.isnan(got[1, :27, 7].view(np.float32)).all()
+    got[1, :27, 7] = clean[1, :27, 7]
+    assert np.array_equal(got, clean)
 
 
 @pytest.mark.parametrize("gp", ["f32", "mixed"])
