@@ -180,8 +180,11 @@ typedef enum p2r_grad_precision { P2R_GRAD_F32 = 0, P2R_GRAD_MIXED = 1, P2R_GRAD
  * ntrk states of 4 bytes (P2R_GRAD_F32) or 8 bytes, plus (stride - 2) * 27 *
  * ntrk values for the recomputed layer inputs of a segment where they do not
  * fit in LDS (stride 8, and stride 4 with F64), of 4 bytes (F32, MIXED) or 8
- * (F64).  A batch whose states of every layer fit 48 MiB of workspace keeps
- * them all, whatever the stride.  The context holds one
+ * (F64).  A batch whose whole workspace at stride 1 (states, ntrk chi2 totals
+ * of the same type, the global sums' partials, 112 * ntrk bytes with MIXED) is
+ * at most 48 MiB runs at stride 1, whatever the stride asked for; a larger
+ * batch makes the context hold at least 48 MiB, so that after it no smaller
+ * one allocates (as a stream capture requires).  The context holds one
  * workspace: adjoint calls on one context must not overlap in time (issue
  * them on one stream, or synchronize between streams or threads).
  * trk_out must not overlap trk_in (the reverse sweep rereads the input
@@ -221,7 +224,8 @@ int p2r_forward_adjoint(p2r_ctx* ctx, const void* trk_in, const void* hits, void
  * P2R_NOALLOC_SCRATCH_BYTES that the library holds on every GPU it runs on
  * until the process ends (its address is resolved once per device at
  * p2r_create); the call itself allocates nothing.  A call that needs more
- * scratch returns P2R_ERR_SHAPE and launches nothing.  Scratch of a call:
+ * scratch returns P2R_ERR_SHAPE and launches nothing.  Scratch of a call, at
+ * the stride that p2r_forward_adjoint would run it at (1 up to 48 MiB):
  * (ceil(nlayer/stride) - 1) * 27 * ntrk checkpoint states plus ntrk chi2
  * totals, of 4 bytes (P2R_GRAD_F32) or 8, plus 8 * (4*nlayer + 1) *
  * ceil(ntrk/256) bytes when grad_global is requested, each part rounded up to

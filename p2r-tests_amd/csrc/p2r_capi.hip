@@ -1383,6 +1383,9 @@ struct AdjointPlan {
   // workspace: checkpoints | chi2 totals | partials | segment store (when not in LDS) | the MIXED tail's
   // hand-over (the adjoint state at layer kTailLayers, 28 floats per track)
   size_t ck_bytes = 0, c2_bytes = 0, part_bytes = 0, seg_bytes = 0, bar_bytes = 0, ws_bytes = 0, lds = 0;
+  // what the context's workspace is grown to: also enough for every smaller batch, which below the line keeps all states
+  // and can need more than this call
+  size_t reserve_bytes = 0;
   p2r_params p{};
 };
 
@@ -1431,7 +1434,9 @@ int adjoint_plan(p2r_ctx* c, const void* trk_in, const void* hits, const void* t
                   ck_bytes_aligned(pl.seg_bytes) + pl.bar_bytes + 256;
   };
   lay_out(1);
-  if (pl.ws_bytes > kSmallAdjointBytes) lay_out(cs);
+  const bool all_states = pl.ws_bytes <= kSmallAdjointBytes;
+  if (!all_states) lay_out(cs);
+  pl.reserve_bytes = all_states ? pl.ws_bytes : std::max(pl.ws_bytes, kSmallAdjointBytes);
   pl.lds = global ? (size_t)(kAdjThreads / 64) * pl.nglob * sizeof(double) : 0;
   return P2R_OK;
 }
@@ -1726,8 +1731,8 @@ int p2r_forward_adjoint(p2r_ctx* c, const void* trk_in, const void* hits, void* 
                               grad_global != nullptr, pl);
   if (rc != P2R_OK || pl.n == 0) return rc;
   DeviceGuard g(c->device);
-  char* ws = static_cast<char*>(c->workspace(pl.ws_bytes));
-  if (!ws) return c->fail(P2R_ERR_NOMEM, "workspace of %zu bytes", pl.ws_bytes);
+  char* ws = static_cast<char*>(c->workspace(pl.reserve_bytes));
+  if (!ws) return c->fail(P2R_ERR_NOMEM, "workspace of %zu bytes", pl.reserve_bytes);
   return adjoint_enqueue(c, pl, trk_in, hits, trk_out, chi2, grad_par, grad_hits, grad_kfact, grad_global, ws,
                          static_cast<hipStream_t>(stream));
 }

@@ -51,3 +51,46 @@ def test_strides_agree_across_the_workspace_line(ctx, gp, tol):
                     ok = np.isfinite(y)
                     assert np.array_equal(ok, np.isfinite(x))
                     assert np.linalg.norm((x - y)[ok]) <= tol * np.linalg.norm(y[ok]), stride
+
+
+@pytest.mark.parametrize("gp", ["f32", "mixed", "f64"])
+def test_a_context_warmed_with_its_largest_batch_allocates_no_more(gp):
+    """A batch below the line keeps every layer's state and so can need more workspace than a larger one above it: the
+    larger one's call reserves that too, so that no smaller batch makes the context allocate, which a stream capture
+    would not allow."""
+    import p2r_amd
+    ctx = p2r_amd.Context(0)
+    n = LARGE
+    trk, hits = p2r_amd.gen_uniform(Shape(1, n, NL, BS))
+    dt, dh = torch.from_numpy(trk).cuda(), torch.from_numpy(hits).cuda()
+    out, chi2 = torch.empty_like(dt), torch.empty(n, device="cuda")
+    gg = torch.empty(4 * NL + 1, device="cuda", dtype=torch.float64)
+
+    def call(m):
+        ctx.forward_adjoint(dt, dh, out, Shape(1, m // BS * BS, NL, BS), grad_precision=gp, checkpoint_stride=4, chi2=chi2,
+                            grad_global=gg)
+
+    call(n)
+    torch.cuda.synchronize()
+    free = torch.cuda.mem_get_info()[0]
+    sizes = (24000, 22000, 12100, 11900, 5000, 64)
+    for m in sizes:
+        call(m)
+        torch.cuda.synchronize()
+        assert torch.cuda.mem_get_info()[0] == free, m
+    # and under capture, which refuses an allocation
+    for m in sizes[1:4]:
+        call(m)
+        want = [t.clone() for t in (out, chi2, gg)]
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g):
+            call(m)
+        for _ in range(3):
+            for t in (out, chi2, gg):
+                t.fill_(float("nan"))
+            g.replay()
+            torch.cuda.synchronize()
+            k = m // BS * BS
+            for a, b, c in ((out, want[0], 28 * k), (chi2, want[1], k), (gg, want[2], gg.numel())):
+                assert torch.equal(a[:c].view(torch.uint8), b[:c].view(torch.uint8)), m
+    ctx.close()
