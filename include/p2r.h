@@ -303,13 +303,17 @@ int p2r_graph_destroy(p2r_graph* graph);
  * templates the kernel on <bsize, layers>).  Here they are runtime choices held
  * by the context, set by hand or measured by the autotuners below. */
 typedef struct p2r_tuning {
-  int32_t fwd_threads;           /* workgroup size of p2r_forward: 64, 128 or 256 (default 256) */
+  int32_t fwd_threads;           /* workgroup size of p2r_forward: 64, 128 or 256 (default 256).  Neither this nor
+                                    fwd_waves matters to P2R_REFERENCE batches of at most 512 tracks per compute
+                                    unit (131 072 on an MI355X) with all layers in one launch, whose layers are
+                                    dealt to wavefronts of their own */
   int32_t fwd_layers_per_launch; /* 0 = all layers in one launch (default); n = launches of n layers,
                                     the state passing through trk_out in between */
   int32_t ragged_schedule;       /* what P2R_RAGGED_AUTO runs: P2R_RAGGED_PAIR_STREAM (default),
                                     P2R_RAGGED_LAYER_ORDER, 1, 2, 4 */
   int32_t ragged_threads;        /* workgroup size of the layer-ordered schedule: 64, 128 or 256 (256) */
-  int32_t checkpoint_stride;     /* what checkpoint_stride = 0 means in p2r_forward_adjoint: 1, 2, 4, 8 (4) */
+  int32_t checkpoint_stride;     /* what checkpoint_stride = 0 means in p2r_forward_adjoint: 1, 2, 4, 8 (4);
+                                    batches of at most 48 MiB of workspace at stride 1 run at 1 */
   int32_t fwd_waves;             /* register budget of the p2r_forward kernels, in waves per SIMD:
                                     0 = the library's choice (default: 3 for P2R_EXACT, 4 for
                                     P2R_FAST), 1 = the compiler's allocation, 3 or 4 (fewer
@@ -341,7 +345,10 @@ typedef struct p2r_tune_report {
  *            best of those;
  *   ragged:  ragged_schedule {layer order x ragged_threads {64, 128, 256},
  *            pair stream, sorted tiles of 1, 2, 4 rounds};
- *   adjoint: checkpoint_stride {1, 2, 4, 8} (grad_precision as given). */
+ *   adjoint: checkpoint_stride {1, 2, 4, 8} (grad_precision as given).
+ * Candidates that run the same kernels on this batch (see p2r_tuning) are timed
+ * once and reported with that time; if they are the fastest, the tuning keeps
+ * of their choices the one it had. */
 int p2r_autotune_forward(p2r_ctx* ctx, const void* trk_in, const void* hits, void* trk_out, const p2r_shape* shape,
                          int semantics, const p2r_params* params, int32_t reps, p2r_tune_report* report,
                          void* stream);

@@ -1389,6 +1389,28 @@ struct AdjointPlan {
   p2r_params p{};
 };
 
+// The stride that a call of pl.n > 0 tracks runs at (`asked`, or 1 below the line above) and its workspace.
+void lay_out_adjoint(AdjointPlan& pl, int asked, bool global) {
+  pl.nglob = 4 * pl.nlayer + 1;
+  pl.grid = grid_for_n(pl.n, kAdjThreads);
+  auto lay_out = [&](int stride) {
+    pl.cs = stride;
+    const size_t n = pl.n, sz = pl.grad_precision == P2R_GRAD_F32 ? sizeof(float) : sizeof(double);
+    const size_t nck = (size_t)((pl.nlayer + stride - 1) / stride - 1);
+    pl.ck_bytes = std::max<size_t>(nck, 1) * 27 * n * sz;
+    pl.c2_bytes = n * sz;
+    pl.part_bytes = global ? (size_t)pl.grid * pl.nglob * sizeof(double) : 0;
+    pl.seg_bytes = seg_global_bytes(pl.grad_precision, stride, n);
+    pl.bar_bytes = pl.grad_precision == P2R_GRAD_MIXED ? (size_t)28 * sizeof(float) * n : 0;
+    pl.ws_bytes = ck_bytes_aligned(pl.ck_bytes) + ck_bytes_aligned(pl.c2_bytes) + ck_bytes_aligned(pl.part_bytes) +
+                  ck_bytes_aligned(pl.seg_bytes) + pl.bar_bytes + 256;
+  };
+  lay_out(1);
+  const bool all_states = pl.ws_bytes <= kSmallAdjointBytes;
+  if (!all_states) lay_out(asked);
+  pl.reserve_bytes = all_states ? pl.ws_bytes : std::max(pl.ws_bytes, kSmallAdjointBytes);
+}
+
 int adjoint_plan(p2r_ctx* c, const void* trk_in, const void* hits, const void* trk_out, const p2r_shape* s,
                  const p2r_params* params, int grad_precision, int32_t checkpoint_stride, bool global,
                  AdjointPlan& pl) {
@@ -1416,27 +1438,10 @@ int adjoint_plan(p2r_ctx* c, const void* trk_in, const void* hits, const void* t
   pl.n = (uint32_t)ntrk;
   pl.bs = (uint32_t)s->bsize;
   pl.nlayer = s->nlayer;
-  pl.nglob = 4 * s->nlayer + 1;
   pl.grad_precision = grad_precision;
   pl.p = p;
   if (ntrk == 0) return P2R_OK;
-  pl.grid = grid_for_n(ntrk, kAdjThreads);
-  auto lay_out = [&](int stride) {
-    pl.cs = stride;
-    const size_t sz = grad_precision == P2R_GRAD_F32 ? sizeof(float) : sizeof(double);
-    const size_t nck = (size_t)((pl.nlayer + stride - 1) / stride - 1);
-    pl.ck_bytes = std::max<size_t>(nck, 1) * 27 * ntrk * sz;
-    pl.c2_bytes = ntrk * sz;
-    pl.part_bytes = global ? (size_t)pl.grid * pl.nglob * sizeof(double) : 0;
-    pl.seg_bytes = seg_global_bytes(grad_precision, stride, ntrk);
-    pl.bar_bytes = grad_precision == P2R_GRAD_MIXED ? (size_t)28 * sizeof(float) * ntrk : 0;
-    pl.ws_bytes = ck_bytes_aligned(pl.ck_bytes) + ck_bytes_aligned(pl.c2_bytes) + ck_bytes_aligned(pl.part_bytes) +
-                  ck_bytes_aligned(pl.seg_bytes) + pl.bar_bytes + 256;
-  };
-  lay_out(1);
-  const bool all_states = pl.ws_bytes <= kSmallAdjointBytes;
-  if (!all_states) lay_out(cs);
-  pl.reserve_bytes = all_states ? pl.ws_bytes : std::max(pl.ws_bytes, kSmallAdjointBytes);
+  lay_out_adjoint(pl, cs, global);
   pl.lds = global ? (size_t)(kAdjThreads / 64) * pl.nglob * sizeof(double) : 0;
   return P2R_OK;
 }
@@ -1520,6 +1525,21 @@ int capture_graph(p2r_ctx* c, void* ws, p2r_graph** out, F&& enqueue) {
   return P2R_OK;
 }
 }  // namespace
+
+bool forward_splits_layers(const p2r_ctx& c, const p2r_shape& s, int semantics, int per_launch) {
+  return semantics == P2R_REFERENCE && s.nevts > 0 && s.ntrks > 0 && s.nlayer <= P2R_MAX_NLAYER &&
+         (per_launch <= 0 || per_launch >= s.nlayer) &&
+         split_layers(c.num_cus, (uint64_t)s.nevts * (uint64_t)s.ntrks, s.nlayer, false).waves > 0;
+}
+
+int adjoint_run_stride(const p2r_shape& s, int grad_precision, int stride, bool global) {
+  AdjointPlan pl;
+  pl.n = (uint32_t)((uint64_t)s.nevts * (uint64_t)s.ntrks);
+  pl.nlayer = s.nlayer;
+  pl.grad_precision = grad_precision;
+  if (pl.n > 0) lay_out_adjoint(pl, stride, global);
+  return pl.cs;
+}
 
 // ---------------------------------------------------------------------------
 extern "C" {

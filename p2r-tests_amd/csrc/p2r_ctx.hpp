@@ -101,6 +101,14 @@ struct p2r_ctx {
   }
 };
 
+// What a call runs, for the autotuners, which time only what differs (p2r_capi.hip); shapes as the entry points take them.
+// Whether p2r_forward deals the batch's layers to several wavefronts, which no other launch choice changes.
+__attribute__((visibility("hidden"))) bool forward_splits_layers(const p2r_ctx& c, const p2r_shape& s, int semantics,
+                                                                 int per_launch);
+// The checkpoint stride that p2r_forward_adjoint runs at when asked for `stride`.
+__attribute__((visibility("hidden"))) int adjoint_run_stride(const p2r_shape& s, int grad_precision, int stride,
+                                                             bool global);
+
 // True when the byte ranges [a, a + na) and [b, b + nb) share a byte.
 inline bool overlaps(const void* a, size_t na, const void* b, size_t nb) {
   const char *x = static_cast<const char*>(a), *y = static_cast<const char*>(b);

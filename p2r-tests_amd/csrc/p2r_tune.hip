@@ -60,13 +60,18 @@ int warm_up(p2r_ctx* c, hipStream_t st, const std::function<int()>& call) {
 }
 
 // Times candidate i (selected by set(i)) for i in [0, n) in two interleaved passes and keeps the smaller
-// mean of each; set(i) must leave the context ready for call().
+// mean of each; set(i) must leave the context ready for call().  Candidate i runs the same kernels as candidate
+// same(i) <= i: only first ones are timed, and the others take their time, so that noise ranks no equals.
 int time_candidates(p2r_ctx* c, hipStream_t st, int reps, int n, const std::function<void(int)>& set,
-                    const std::function<int()>& call, float* best_ms) {
+                    const std::function<int(int)>& same, const std::function<int()>& call, float* best_ms) {
   set(0);
   int rc = warm_up(c, st, call);
   for (int pass = 0; rc == P2R_OK && pass < 2; ++pass)
     for (int i = 0; rc == P2R_OK && i < n; ++i) {
+      if (same(i) != i) {
+        best_ms[i] = best_ms[same(i)];
+        continue;
+      }
       set(i);
       float ms = 0.f;
       rc = time_calls(c, st, reps, call, &ms);
@@ -74,16 +79,21 @@ int time_candidates(p2r_ctx* c, hipStream_t st, int reps, int n, const std::func
     }
   return rc;
 }
+int itself(int i) { return i; }
 
 struct Collect {
   p2r_tune_report rep{};
   void add(const p2r_tune_entry& e) {
     if (rep.count < 32) rep.entry[rep.count++] = e;
   }
-  void finish(p2r_tune_report* out) {
+  // Of entries with the same time (candidates that run the same kernels) an entry that `in_force` accepts is the best:
+  // a choice that makes no difference here stays what it was.
+  void finish(p2r_tune_report* out, const std::function<bool(const p2r_tune_entry&)>& in_force = {}) {
     rep.best = 0;
-    for (int i = 1; i < rep.count; ++i)
-      if (rep.entry[i].ms < rep.entry[rep.best].ms) rep.best = i;
+    for (int i = 1; i < rep.count; ++i) {
+      const p2r_tune_entry &e = rep.entry[i], &b = rep.entry[rep.best];
+      if (e.ms < b.ms || (e.ms == b.ms && in_force && in_force(e) && !in_force(b))) rep.best = i;
+    }
     if (out) *out = rep;
   }
 };
@@ -160,21 +170,29 @@ int p2r_autotune_forward(p2r_ctx* c, const void* trk_in, const void* hits, void*
     }
   }
   auto run = [&] { return p2r_forward(c, trk_in, hits, trk_out, s, semantics, params, nullptr, stream); };
+  // the first three (all layers in one launch) run alike where the batch's layers are split
+  const bool split = forward_splits_layers(*c, *s, semantics, 0);
   std::vector<float> ms(cand.size(), 0.f);
-  int rc = time_candidates(c, st, reps, (int)cand.size(), [&](int i) { c->tune = cand[i]; }, run, ms.data());
+  int rc = time_candidates(c, st, reps, (int)cand.size(), [&](int i) { c->tune = cand[i]; },
+                           [&](int i) { return split && i < 3 ? 0 : i; }, run, ms.data());
   if (rc != P2R_OK) {
     c->tune = keep;
     return rc;
   }
   // register budget at the best workgroup size / layer split
-  const size_t b0 = std::min_element(ms.begin(), ms.end()) - ms.begin();
+  size_t b0 = std::min_element(ms.begin(), ms.end()) - ms.begin();
+  const bool no_budget = split && b0 < 3;
+  if (no_budget)
+    for (size_t i = 0; i < 3; ++i)
+      if (cand[i].fwd_threads == keep.fwd_threads) b0 = i;
   for (int waves : {1, 3, 4}) {
     p2r_tuning t = cand[b0];
     t.fwd_waves = waves;
     cand.push_back(t);
   }
-  float wms[3] = {};
-  rc = time_candidates(c, st, reps, 3, [&](int i) { c->tune = cand[cand.size() - 3 + i]; }, run, wms);
+  float wms[3] = {ms[b0], ms[b0], ms[b0]};
+  if (!no_budget)
+    rc = time_candidates(c, st, reps, 3, [&](int i) { c->tune = cand[cand.size() - 3 + i]; }, itself, run, wms);
   c->tune = keep;
   if (rc != P2R_OK) return rc;
   for (float w : wms) ms.push_back(w);
@@ -184,7 +202,9 @@ int p2r_autotune_forward(p2r_ctx* c, const void* trk_in, const void* hits, void*
     e.waves = cand[i].fwd_waves;
     col.add(e);
   }
-  col.finish(report);
+  col.finish(report, [&](const p2r_tune_entry& e) {
+    return e.threads == keep.fwd_threads && e.waves == keep.fwd_waves;
+  });
   const p2r_tuning& b = cand[col.rep.best];
   c->tune.fwd_threads = b.fwd_threads;
   c->tune.fwd_layers_per_launch = b.fwd_layers_per_launch;
@@ -219,6 +239,7 @@ int p2r_autotune_ragged(p2r_ctx* c, const void* trk_in, const void* hits, void* 
         c->tune.ragged_schedule = cand[i].schedule;
         c->tune.ragged_threads = cand[i].threads;
       },
+      itself,
       [&] {
         return p2r_forward_ragged(c, trk_in, hits, trk_out, blk_offsets, nevts, layer_mask, nlayer, bsize, semantics,
                                   params, nullptr, P2R_RAGGED_AUTO, stream);
@@ -252,6 +273,12 @@ int p2r_autotune_adjoint(p2r_ctx* c, const void* trk_in, const void* hits, void*
   float ms[4] = {};
   const int rc = time_candidates(
       c, st, reps, 4, [&](int i) { cs = strides[i]; },
+      [&](int i) {
+        int j = 0;
+        auto runs = [&](int k) { return adjoint_run_stride(*s, grad_precision, strides[k], grad_global != nullptr); };
+        while (j < i && runs(j) != runs(i)) ++j;
+        return j;
+      },
       [&] {
         return p2r_forward_adjoint(c, trk_in, hits, trk_out, s, params, grad_precision, cs, chi2, grad_par,
                                    grad_hits, grad_kfact, grad_global, stream);
@@ -264,7 +291,7 @@ int p2r_autotune_adjoint(p2r_ctx* c, const void* trk_in, const void* hits, void*
     t.checkpoint_stride = strides[i];
     col.add(entry_of(t, s->bsize, ms[i], 0));
   }
-  col.finish(report);
+  col.finish(report, [&](const p2r_tune_entry& e) { return e.checkpoint_stride == c->tune.checkpoint_stride; });
   c->tune.checkpoint_stride = col.rep.entry[col.rep.best].checkpoint_stride;
   return P2R_OK;
 }

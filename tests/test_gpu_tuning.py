@@ -125,6 +125,34 @@ def test_autotune_forward_picks_a_candidate(ctx, orc, batch):
     assert np.array_equal(o, o0) and np.array_equal(c, c0)
 
 
+@pytest.mark.parametrize("threads,waves,stride", [(128, 4, 2), (64, 0, 8), (256, 1, 1)])
+def test_autotuners_do_not_rank_equal_candidates(ctx, batch, threads, waves, stride):
+    """On a batch that every stride runs alike, and whose layers are split whatever the workgroup size and the register
+    budget, those candidates report one time and the tuning keeps the choices it had."""
+    shape, dt, dh = batch
+    do = torch.empty_like(dt)
+    ctx.set_tuning(fwd_threads=threads, fwd_waves=waves, checkpoint_stride=stride)
+    ents = ctx.autotune_adjoint(dt, dh, do, shape, grad_precision="f64", reps=1).as_list()
+    assert len(ents) == 4 and len({e["ms"] for e in ents}) == 1
+    rep = ctx.autotune_forward(dt, dh, do, shape, "reference", reps=2)
+    ents = rep.as_list()
+    one = [e for e in ents if e["layers_per_launch"] == 0]
+    assert len(one) == 6 and len({e["ms"] for e in one}) == 1
+    assert len({e["ms"] for e in ents}) > 1
+    assert ents[rep.best]["layers_per_launch"] == 0  # one launch against two and four
+    t = ctx.get_tuning()
+    assert (t.fwd_threads, t.fwd_layers_per_launch, t.fwd_waves, t.checkpoint_stride) == (threads, 0, waves, stride)
+    # a batch above the lines has every candidate timed
+    import p2r_amd
+    large = Shape(1, 262176, 2, 32)
+    trk, hits = p2r_amd.gen_uniform(large)
+    t, h = torch.from_numpy(trk).cuda(), torch.from_numpy(hits).cuda()
+    o = torch.empty_like(t)
+    assert len({e["ms"] for e in ctx.autotune_adjoint(t, h, o, large, grad_precision="f64", reps=1).as_list()}) > 1
+    # 9 candidates; with the 6 of one launch alike there would be 4 times
+    assert len({e["ms"] for e in ctx.autotune_forward(t, h, o, large, "reference", reps=1).as_list()}) > 4
+
+
 def test_repack_round_trip_and_width_invariance(ctx, batch):
     """32 -> 16 -> 32 restores every word; the forward on the width-16 copy equals the width-32 forward
     after repacking its output back."""
