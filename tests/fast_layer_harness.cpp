@@ -22,7 +22,7 @@
 namespace fst {
 inline double rcp_est(double x) { return 1.0 / x; }
 inline float rcp_prio(float x) { return 1.0f / x; }
-inline float rsq_prio(float x) { return 1.0f / std::sqrt(x); }
+inline float rsq_prio(float x) { return 1.0f / std::sqrt(std::fabs(x) < 1.17549435e-38f ? 0.0f : x); }  // as v_rsq_f32
 inline void opaque(float&) {}
 inline void phase_boundary() {}
 using real = float;
