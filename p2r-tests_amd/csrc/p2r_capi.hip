@@ -156,7 +156,7 @@ __global__ __launch_bounds__(kThreads, MINW) void fwd_uniform_kernel(const float
     Hit h;
     wh.load(l, h);
     Trk prop;
-    float r;
+    typename Lane<EXACT>::Carry carry;
     if (SEM == P2R_REFERENCE) {
       // tbb.cpp:894: every layer starts from the input track.  The barriers, on the input parameters in
       // place and on the covariance column's offset, make every layer recompute and reread it; nothing is
@@ -167,11 +167,11 @@ __global__ __launch_bounds__(kThreads, MINW) void fwd_uniform_kernel(const float
       asm volatile("" : "+v"(col));
       q = q_in;
       k = (float)q * kfact;
-      r = Lane<EXACT>::propagate(in_par, LdsCov{cov_lds + col * 21u}, k, h.pos[0], h.pos[1], prop);
+      carry = Lane<EXACT>::propagate(in_par, LdsCov{cov_lds + col * 21u}, k, h.pos[0], h.pos[1], prop);
     } else {
-      r = Lane<EXACT>::propagate(cur.par, cur.cov, k, h.pos[0], h.pos[1], prop);  // propagate-tor-test_hip.cu:842-845
+      carry = Lane<EXACT>::propagate(cur.par, cur.cov, k, h.pos[0], h.pos[1], prop);  // propagate-tor-test_hip.cu:842-845
     }
-    float c = Lane<EXACT>::update(prop, h, r);
+    float c = Lane<EXACT>::update(prop, h, carry);
     if (opts) apply_options<EXACT>(opts, prop, q, k, kfact);
     if (SEM == P2R_REFERENCE) {
       // Only the last layer's result is returned in reference semantics; the
@@ -243,8 +243,8 @@ __global__ __launch_bounds__(1024) void fwd_layers_kernel(const float* trk, cons
       q = q_in;
       float k = (float)q * kfact;
       Trk prop;
-      const float r = Lane<EXACT>::propagate(in_par, LdsCov{cov_lds + col * 21u}, k, h.pos[0], h.pos[1], prop);
-      float c = Lane<EXACT>::update(prop, h, r);
+      const auto carry = Lane<EXACT>::propagate(in_par, LdsCov{cov_lds + col * 21u}, k, h.pos[0], h.pos[1], prop);
+      float c = Lane<EXACT>::update(prop, h, carry);
       if (opts) apply_options<EXACT>(opts, prop, q, k, kfact);
       opaque(prop);
       opaque(c);
@@ -316,8 +316,8 @@ __device__ __forceinline__ void ragged_slot(const float* __restrict__ trk, const
       src = cur;
     }
     Trk prop;
-    const float r = Lane<EXACT>::propagate(src.par, src.cov, k, h.pos[0], h.pos[1], prop);
-    float c = Lane<EXACT>::update(prop, h, r);
+    const auto carry = Lane<EXACT>::propagate(src.par, src.cov, k, h.pos[0], h.pos[1], prop);
+    float c = Lane<EXACT>::update(prop, h, carry);
     if (opts) apply_options<EXACT>(opts, prop, q, k, kfact);
     if (SEM == P2R_REFERENCE) {
       opaque(prop);
@@ -463,8 +463,8 @@ __global__ __launch_bounds__(kThreads) void fwd_ragged_layer_kernel(const float*
         src = cur;
       }
       Trk prop;
-      const float r = Lane<EXACT>::propagate(src.par, src.cov, k, h.pos[0], h.pos[1], prop);
-      float c = Lane<EXACT>::update(prop, h, r);
+      const auto carry = Lane<EXACT>::propagate(src.par, src.cov, k, h.pos[0], h.pos[1], prop);
+      float c = Lane<EXACT>::update(prop, h, carry);
       if (opts) apply_options<EXACT>(opts, prop, q, k, kfact);
       if (SEM == P2R_REFERENCE) {
         opaque(prop);
@@ -634,8 +634,8 @@ __global__ __launch_bounds__(64 * kPsWaves) void fwd_ragged_stream_kernel(const 
       float k = (float)q * kfact;
       if (SEM == P2R_REFERENCE) opaque(src);
       Trk prop;
-      const float r = Lane<EXACT>::propagate(src.par, src.cov, k, h.pos[0], h.pos[1], prop);
-      float cc = Lane<EXACT>::update(prop, h, r);
+      const auto carry = Lane<EXACT>::propagate(src.par, src.cov, k, h.pos[0], h.pos[1], prop);
+      float cc = Lane<EXACT>::update(prop, h, carry);
       if (opts) apply_options<EXACT>(opts, prop, q, k, kfact);
       if (SEM == P2R_REFERENCE) {
         opaque(prop);
@@ -716,7 +716,7 @@ template <class R, bool EXACT> struct MathOf;
 template <> struct MathOf<float, true> {
   using T = exact::Trk; using H = exact::Hit;
   static __device__ __forceinline__ float fwd(const T& in, float k, const H& h, T& out) {
-    return exact::kalman_update_r(out, h, exact::propagate_to_r(in, k, h.pos[0], h.pos[1], out));
+    return exact::kalman_update_c(out, h, exact::propagate_to_r(in, k, h.pos[0], h.pos[1], out));
   }
   static __device__ __forceinline__ void adj(const T& in, float k, const H& h, T& bar, float& kb, float hb[3]) {
     exact::layer_adjoint(in, k, h, bar, kb, hb);
@@ -734,7 +734,7 @@ template <> struct MathOf<float, false> {
 template <bool EXACT> struct MathOf<double, EXACT> {
   using T = dbl::Trk; using H = dbl::Hit;
   static __device__ __forceinline__ double fwd(const T& in, double k, const H& h, T& out) {
-    return dbl::kalman_update_r(out, h, dbl::propagate_to_r(in, k, h.pos[0], h.pos[1], out));
+    return dbl::kalman_update_c(out, h, dbl::propagate_to_r(in, k, h.pos[0], h.pos[1], out));
   }
   static __device__ __forceinline__ void adj(const T& in, double k, const H& h, T& bar, double& kb, double hb[3]) {
     dbl::layer_adjoint(in, k, h, bar, kb, hb);
@@ -809,7 +809,7 @@ __global__ __launch_bounds__(kAdjThreads, MINW) void adjoint_fwd_kernel(
 #pragma unroll
       for (int f = 0; f < 21; ++f) cp[(size_t)(6 + f) * ntrk] = cur.cov[f];
     }
-    HitT<RS> h;  // loaded as the layer starts (no prefetch: 125 VGPRs in exact FP32, 4 waves)
+    HitT<RS> h;  // loaded as the layer starts (no prefetch: 124 VGPRs in exact FP32, 4 waves)
     load_hit_as(hb + l * hstride, bs, h);
     TrkT<RS> nxt;
     c2 += MS::fwd(cur, (RS)k, h, nxt);
@@ -1182,7 +1182,7 @@ template <int SEM, bool CHI2, bool EXACT>
 void launch_uniform_e(int waves, dim3 grid, dim3 block, hipStream_t st, const UniformLaunch& a, const float* in,
                       int l0, int l1, bool acc) {
   // 0 = the library's choice: the 3-wave budget for the exact instance, 4 waves for the fast one.  At every
-  // budget the exact kernels fit 4 waves per SIMD (97-127 VGPRs) and the fast ones 5 or 6 (73-92), without
+  // budget the exact kernels fit 4 or 5 waves per SIMD (96-128 VGPRs) and the fast ones 5 or 6 (73-92), without
   // spills, and run alike within noise; the choice stays for the autotuner.
   if (waves == 0) waves = EXACT ? 3 : 4;
   if (waves == 3) launch_uniform_w<SEM, CHI2, EXACT, 3>(grid, block, st, a, in, l0, l1, acc);

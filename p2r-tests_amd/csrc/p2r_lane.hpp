@@ -125,28 +125,30 @@ using Jac = JacT<real>;
 }  // namespace dbl
 
 // Compile-time selection of the instance.  propagate returns what the update of the same layer needs of it: the
-// hit's radius (exact), its reciprocal (fast).
+// tangent plane's rotation (exact), the reciprocal of the hit's radius (fast).
 template <bool EXACT> struct Lane;
 template <> struct Lane<true> {
+  using Carry = exact::Carry;
   template <class PC>
-  static __device__ __forceinline__ float propagate(const float (&par)[6], const PC& P, float k, float hx, float hy,
+  static __device__ __forceinline__ Carry propagate(const float (&par)[6], const PC& P, float k, float hx, float hy,
                                                     Trk& out) {
     return exact::propagate_to_r_c(par, P, k, hx, hy, out);
   }
-  static __device__ __forceinline__ float update(Trk& t, const Hit& h, float r) {
-    return exact::kalman_update_r(t, h, r);
+  static __device__ __forceinline__ float update(Trk& t, const Hit& h, Carry c) {
+    return exact::kalman_update_c(t, h, c);
   }
   static __device__ __forceinline__ float update(Trk& t, const Hit& h) { return exact::kalman_update(t, h); }
   static __device__ __forceinline__ float wrap_phi(float phi) { return exact::m_wrap_phi(phi); }
 };
 template <> struct Lane<false> {
+  using Carry = float;
   template <class PC>
   static __device__ __forceinline__ float propagate(const float (&par)[6], const PC& P, float k, float hx, float hy,
                                                     Trk& out) {
     return fast::fast_propagate(par, P, k, hx, hy, out);
   }
-  static __device__ __forceinline__ float update(Trk& t, const Hit& h, float r) {
-    return fast::fast_update(t, h, r);
+  static __device__ __forceinline__ float update(Trk& t, const Hit& h, float rinv) {
+    return fast::fast_update(t, h, rinv);
   }
   static __device__ __forceinline__ float wrap_phi(float phi) { return fast::m_wrap_phi(phi); }
 };
