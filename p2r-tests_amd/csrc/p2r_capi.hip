@@ -711,7 +711,7 @@ constexpr int kAdjThreads = 256;
 
 template <class R, bool EXACT> struct MathOf;
 // fwd: one layer of the forward pass (the updated state and its chi2): p2r_forward's own per-lane code
-// (propagate_to_r, kalman_update) in the instance's arithmetic, shared by the adjoint's forward pass, the
+// (propagate_to_r and kalman_update_c; the fast instance's fast_propagate and fast_update), shared by the adjoint's forward pass, the
 // reverse sweep's segment recompute and the FP64 tail.
 template <> struct MathOf<float, true> {
   using T = exact::Trk; using H = exact::Hit;
