@@ -145,8 +145,9 @@ def test_adjoint_fp32_gradients_vs_fp64(orc, ctx, batch, gp, precision, median_b
 
 
 def test_checkpoint_stride_does_not_change_gradients(ctx, batch):
-    """Exact FP32: the segments' recomputed inputs are the forward pass's states bit for bit (no contraction,
-    so both kernels round every operation alike), and the gradients are the same words at every stride."""
+    """Exact FP32: the gradients are the same words at every stride asked for.  This batch keeps every layer's state
+    whatever the stride; above that line, where the segments' recomputed inputs are the forward pass's states bit
+    for bit (no contraction, so both kernels round every operation alike), test_gpu_adjoint_strides.py tests it."""
     shape, trk, hits = batch
     ref = run_adjoint(ctx, trk, hits, shape, "f32", cs=4)[2]
     for cs in (1, 2, 8):
@@ -156,7 +157,8 @@ def test_checkpoint_stride_does_not_change_gradients(ctx, batch):
 
 @pytest.mark.parametrize("gp,precision,tol", [("f32", "fast", 1.5e-2), ("mixed", "exact", 1e-5), ("f64", "exact", 1e-8)])
 def test_checkpoint_stride_with_fused_arithmetic(ctx, batch, gp, precision, tol):
-    """Where the recompute fuses multiply-adds (fast FP32, and the FP64 states of MIXED and F64), the
+    """(This batch keeps every layer's state whatever the stride; test_gpu_adjoint_strides.py has the larger ones.)
+    Where the recompute fuses multiply-adds (fast FP32, and the FP64 states of MIXED and F64), the
     compiler fuses them per kernel, so the forward pass and a segment's recompute may round a state
     differently in its last bit; the gradients then agree across strides to the arithmetic's precision
     (normwise per track), not word for word.  The chained fit's ill-conditioned updates amplify a last-bit

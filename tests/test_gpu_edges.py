@@ -107,8 +107,9 @@ def test_hit_on_the_z_axis_has_no_finite_result(ctx, semantics, precision, ntrks
 @pytest.mark.parametrize("gp", ["f32", "mixed"])
 @pytest.mark.parametrize("nlayer", [1, 3])
 def test_adjoint_short_fits_all_strides(ctx, nlayer, gp):
-    """nlayer below the checkpoint stride: every stride gives the same gradients, and the FP32 forward
-    outputs equal p2r_forward's.  With mixed and one layer the FP32 sweep has nothing to do: the FP64
+    """nlayer below the checkpoint stride: every stride asked for gives the same gradients, and the FP32 forward
+    outputs equal p2r_forward's (every state kept, as this batch is small; each stride's own kernels:
+    test_gpu_adjoint_strides.py).  With mixed and one layer the FP32 sweep has nothing to do: the FP64
     reverse of the first two layers takes all of it."""
     import p2r_amd
     shape = Shape(1, 1024, nlayer, 32)
@@ -138,9 +139,9 @@ def test_adjoint_short_fits_all_strides(ctx, nlayer, gp):
 @pytest.mark.parametrize("gp,cs", [("f32", 4), ("f32", 8), ("f64", 4), ("mixed", 4)])
 def test_adjoint_batch_ending_inside_a_workgroup(ctx, gp, cs):
     """A batch of 1000 tracks (the last 256-lane workgroup 24 lanes short) gives each track the same words
-    as the same tracks inside a batch of 1024.  Covers the segment states in LDS (FP32, stride 4) and in
+    as the same tracks inside a batch of 1024, every state kept.  Segment states in LDS (FP32, stride 4) and in
     the workspace (FP32 stride 8, FP64 stride 4), where the lanes past the batch share the last track's
-    slots."""
+    slots, take the larger batches of test_gpu_adjoint_strides.py."""
     import p2r_amd
     bs, nl = 8, 20
     big, small = Shape(1, 1024, nl, bs), Shape(1, 1000, nl, bs)
