@@ -101,6 +101,25 @@ def test_launch_choices_are_bit_identical(ctx, batch, sem):
             assert np.array_equal(o, o0) and np.array_equal(c, c0), (waves, prec)
 
 
+@pytest.mark.parametrize("precision", ["exact", "fast"])
+def test_launch_choices_are_bit_identical_above_the_layer_split(ctx, orc, precision):
+    """The same in reference semantics on a batch whose layers are not split, where workgroup size and register budget
+    reach the kernel."""
+    import p2r_amd
+    shape = Shape(1, 131104, 4, 32)
+    trk, hits = p2r_amd.gen_uniform(shape)
+    dt, dh = torch.from_numpy(trk).cuda(), torch.from_numpy(hits).cuda()
+    ref_o, ref_c = _fwd(ctx, dt, dh, shape, "reference", precision)
+    if precision == "exact":
+        want_o, want_c = _oracle_words(orc, dt, dh, shape, "reference")
+        assert _equal_words(ref_o, want_o) and _equal_words(ref_c, want_c)
+    for choice in ({"fwd_threads": 64}, {"fwd_threads": 128}, {"fwd_waves": 1}, {"fwd_waves": 3}, {"fwd_waves": 4},
+                   {"fwd_layers_per_launch": 3}, {"fwd_threads": 128, "fwd_waves": 4, "fwd_layers_per_launch": 1}):
+        ctx.set_tuning(**{"fwd_threads": 256, "fwd_waves": 0, "fwd_layers_per_launch": 0, **choice})
+        o, c = _fwd(ctx, dt, dh, shape, "reference", precision)
+        assert _equal_words(o, ref_o) and _equal_words(c, ref_c), choice
+
+
 def test_autotune_forward_picks_a_candidate(ctx, orc, batch):
     shape, dt, dh = batch
     do = torch.empty_like(dt)
