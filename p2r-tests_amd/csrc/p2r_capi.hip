@@ -201,9 +201,9 @@ __global__ __launch_bounds__(kThreads, MINW) void fwd_uniform_kernel(const float
 // covariance waits in LDS for all of them, and the last layer's wavefront writes the track, after the barrier
 // that follows the workgroup's reads of it.  The chi2 sum over a track's layers is taken in layer order from LDS,
 // so it needs all the layers in one workgroup (gridDim.y == 1), as does trk_out over trk_in.
-// Bound by the latency of a wavefront's layers: with one wavefront per tile, an event's 150 took 50.5 us (exact, 9600
+// Bound by the latency of a wavefront's layers: with one wavefront per tile, an event's 150 take 53.7 us (exact, 9600
 // tracks x 20 layers) on 150 of the 1024 SIMDs, a layer after the other at an instruction per 4.3 cycles; with the
-// layers dealt out it takes 10.9, most of which is the launch.
+// layers dealt out 8.0, most of which is the call.
 constexpr int kTileTracks = 64;
 template <bool CHI2, bool EXACT>
 __global__ __launch_bounds__(1024) void fwd_layers_kernel(const float* trk, const float* __restrict__ hits, float* out,
@@ -1202,8 +1202,9 @@ struct LayerSplit {
 };
 LayerSplit split_layers(int num_cus, uint64_t ntrk, int nlayer, bool one_group) {
   // The line: from 2 wavefronts per SIMD on (4 SIMDs a CU) fwd_uniform_kernel fills the issue slots by itself.
-  // Exact x 20 layers, split against not, us: 512 tiles 18.7 / 51.6, 1024 31.2 / 52.9, 1500 53.0 / 58.3, 2048 60.7 /
-  // 60.8; beyond that a static division only adds imbalance.
+  // x 20 layers, split against not, us: exact 512 tiles 18.7 / 54.1, 1024 30.8 / 55.1, 1500 50.6 / 56.5, 2048 58.9 /
+  // 62.6, fast 12.1 / 33.1, 19.4 / 35.6, 31.2 / 39.3, 38.7 / 40.5; beyond that a static division adds imbalance: 2500
+  // tiles 86.7 / 89.8 exact but 53.2 / 52.3 fast, 3000 105.3 / 92.6 and 57.9 / 56.9.
   const uint64_t tiles = (ntrk + kTileTracks - 1) / kTileTracks, simds = (uint64_t)num_cus * 4;
   LayerSplit s;
   if (nlayer < 2 || tiles > 2 * simds) return s;
@@ -1368,11 +1369,13 @@ int resolve_scratch(int device, void** out) {
   return P2R_OK;
 }
 
-// A batch whose states of every layer fit this much workspace keeps them all, whatever the checkpoint stride: it is
-// bound by the latency of its few wavefronts, and recomputing a segment's states from its checkpoint only lengthens
-// them.  9600 tracks x 20 layers (38 MB of FP64 states) at stride 4, us: F64 202 -> 173, 2048 tracks MIXED
-// through autograd 192 -> 184.  Larger batches hide the recompute and would pay for the states' traffic (960 000 tracks
-// MIXED: 2.25 ms at stride 4, 2.45 at stride 1).
+// A batch whose workspace with the states of every layer is at most this keeps them all, whatever the checkpoint stride:
+// it is bound by the latency of its few wavefronts, and recomputing a segment's states from its checkpoint only
+// lengthens them.  Kept against stride 4, 20 layers, us: 2048 tracks F32 134 / 167, MIXED 147 / 164, F64 157 / 189;
+// at the line F32 (24 000 tracks) 152 / 185, MIXED (12 000) 168 / 173, F64 174 / 200.  The line is one of memory: every
+// request that the 64 MiB of p2r_forward_adjoint_noalloc held must fit, and a larger batch's stride is its caller's
+// choice of memory.  In time the states stay ahead to about 64 000 tracks in MIXED (195 / 194; 160 000: 482 / 458) and
+// beyond 256 000 in F32 (437 / 466) and F64 (806 / 883).
 constexpr size_t kSmallAdjointBytes = 48u << 20;
 
 // Validated arguments and workspace layout of one adjoint call.
