@@ -17,7 +17,7 @@ def test_fast_layer_against_the_formulas_in_fp64(tmp_path):
     assert not cases, "an output is finite in one arithmetic only"
     par, cov = (float(v) for v in last.split()[1:])
     print(f"max difference over the propagated sigma: parameters {par:.1e}, covariance {cov:.1e}", flush=True)
-    # z reaches 60 with an ulp of 4e-6 and is summed from two terms; its propagated sigma is 4e-3 and more
+    # x has the smallest propagated sigma, 4e-3 and more, and an ulp of 2e-6 at up to 20: four ulps over five steps
     assert par < 2e-3
     # a term of J P J^T is up to 10 times its sum (j00 = 1 + U g0 all but cancels) at 2^-24 each, over 20 products
     assert cov < 2e-3
